@@ -189,7 +189,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(MIXED && 
             }
         }
         waveLdsSync();
-        double rhoi = 0, gradhi = 0;   // plain: sum E, sum G (kernED); mixed: sum V, sum q D
+        double rhoi = 0, gradhi = 0;   // plain: sum V, sum G (kernVGD); mixed: sum V, sum q D
         G divs = 0, dv[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0}, da[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
         G rxx = 0, rxy = 0, rxz = 0, ryy = 0, ryz = 0, rzz = 0;
         auto keep = [&](int jl) {
@@ -260,12 +260,12 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(MIXED && 
             sep(k, dx, dy, dz);
             // one root for q = r / h and 1 / (r + eps) = (1/r) (1 - eps / r), the next term of order
             // (eps / r)^2; 2^-900 keeps the self pair (whose dx and D are zero) off zero
-            double rij, rinv, E, D;
+            double rij, rinv, V, G0, D;
             sqrtAndInverse(dx * dx + dy * dy + dz * dz + 0x1p-900, rij, rinv);
             const double q = fmin(rij * hinvi, kRad);
-            kernED<double>(q, E, D);
-            rhoi += E;
-            gradhi += fma(q, D, -kGe * E);
+            kernVGD<double>(q, V, G0, D);
+            rhoi += V;
+            gradhi += G0;
             const double rg = fma(-2.220446049250313e-16 * rinv, rinv, rinv) * (-kGp * D);
             const double rx = dx * rg * pmass, ry = dy * rg * pmass, rz = dz * rg * pmass;
             const double dvx = vxi - tj[3][k], dvy = vyi - tj[4][k], dvz = vzi - tj[5][k];
@@ -327,7 +327,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(MIXED && 
         if (!has || sub != 0) continue;
 
         const double hi1 = 1.0 / hi_, hi31 = hi1 * hi1 * hi1, hi41 = hi31 * hi1;
-        double wsum = kWw * ((1.0 - kGe) * rhoi - gradhi), gsum = (kGp + kGw) * gradhi;
+        double wsum = kWw * rhoi, gsum = (kGp + kGw) * gradhi;
         if constexpr (MIXED)
         {
             // brackets to sums, the q of every pair short by (1 + eps/2): as particleSums in nr.hip

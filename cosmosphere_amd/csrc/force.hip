@@ -81,8 +81,10 @@ __device__ inline double pressureOf(double pro2, double rho)
 // unchanged (for g = 1 even their order; the survivors fill the tiles in list order).  On the
 // 16M-particle Plummer mixture the particle test halves the candidates (11.1 to 5.5 per pair).
 //
-// Pair terms: both kernel gradients as truncated powers (the D of kernED) with q cut off at R, so
-// that a side beyond its support adds zeros without a branch, and one root for r and 1/r.  The tile
+// Pair terms: both kernel gradients (the D of kernED) without a branch, q cut off at R, so
+// that a side beyond its support adds zeros, and one root for r and 1/r.  Both sides' terms share
+// one sum per component, kept per tile: over the whole list its rounding errors would be up to 1.4
+// times those of a sum for each side.  The tile
 // holds what the pair needs of j; the pressure and the conductivity factor are taken from rho,
 // 1/rho and p/rho^2 rather than gathered (15 fields instead of 18).  The open instances fit four
 // wavefronts per SIMD (128 VGPRs, 9 KB of LDS each): the chunk's positions are read from their
@@ -113,7 +115,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(PER ? 1 :
         const int iLeaf = a;
         const uint32_t lo = A.jOffset[a], hi = A.jOffset[a + 1];
         const DBox box = A.boxes[A.leafSet[iLeaf]];
-        const double pmass = A.pmass, beta = A.beta, auc = 0.5 * A.pmass * A.alphau;
+        const double pmass = A.pmass, beta = A.beta, auc = 0.5 * A.alphau;
         for (uint32_t q0 = p0; q0 < p1; q0 += kWave)
         {
             const int c = __builtin_amdgcn_readfirstlane((int)min((uint32_t)kWave, p1 - q0));
@@ -197,7 +199,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(PER ? 1 :
                 const double rj2 = DISC ? reachOf(tf[R2][k]) : tf[R2][k];
                 return (dr2 > 0.0) && (dr2 < fmax(reach2, rj2));
             };
-            auto pair = [&](int k) {
+            auto pair = [&](int k, double& px, double& py, double& pz) {
                 double dx, dy, dz;
                 sep(k, dx, dy, dz);
                 const double dr2 = dx * dx + dy * dy + dz * dz;
@@ -236,10 +238,10 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(PER ? 1 :
                 kernED<double>(fmin(qj, kRad), E, Dj);
                 const double di = -kGp * Di;
                 const double gi = di * gki, gj = -kGp * Dj * tf[GK][k];
-                const double f = pmass * ((pro2i + qr2i) * gi + (pro2j + qr2j) * gj);
-                sx -= f * rx; sy -= f * ry; sz -= f * rz;
+                const double f = (pro2i + qr2i) * gi + (pro2j + qr2j) * gj;
+                px -= f * rx; py -= f * ry; pz -= f * rz;
                 divs += di * projv;
-                const double e = pmass * projv * gi;
+                const double e = projv * gi;
                 if constexpr (FULL) f4s += e * (pro2i + heat);
                 else
                 {
@@ -261,12 +263,14 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(PER ? 1 :
                 int t = 0;
                 for (int k = sub; k < nt; k += g, ++t)
                     if (accepts(k)) accept |= 1ull << t;
+                double px = 0, py = 0, pz = 0;   // the tile's sums: shorter chains, smaller errors
                 while (accept)
                 {
                     const int tt = __builtin_ctzll(accept);
                     accept &= accept - 1;
-                    pair(sub + tt * g);
+                    pair(sub + tt * g, px, py, pz);
                 }
+                sx += px; sy += py; sz += pz;
             };
             forEachTileCompact(segStart, segJ, tileHead, jq, A.layout, A.jList, lo, hi, keep, keepJ, load, consume);
             // group sums (and the max of vsigmax): a tree over lanes sub .. g - 1 of each group
@@ -284,8 +288,8 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(PER ? 1 :
             }
             if (has && sub == 0)
             {
-                A.fx[i] = sx; A.fy[i] = sy; A.fz[i] = sz;
-                A.f4[i] = f4s; A.vsig[i] = vmax;
+                A.fx[i] = pmass * sx; A.fy[i] = pmass * sy; A.fz[i] = pmass * sz;
+                A.f4[i] = pmass * f4s; A.vsig[i] = vmax;
                 A.divv[i] = -(pmass * divs) * A.divfac[i];
                 nAcc += (unsigned long long)acc;
                 nCand += cand;
