@@ -117,6 +117,14 @@ __device__ inline double xiLimiter(const double g[9])
     return (fac + tr > 2.220446049250313e-16) ? fac / (fac + tr) : 1.0;
 }
 
+// The reference's guard of 1 / (r + eps), and whether 2^-480 <= r < 2^-25 (by the exponent word).
+constexpr double kEps = 2.220446049250313e-16;
+__device__ inline bool nearEps(double r)
+{
+    constexpr uint32_t lo = (1023u - 480u) << 20, hi = (1023u - 25u) << 20;
+    return (uint32_t)(__double_as_longlong(r) >> 32) - lo < hi - lo;
+}
+
 // One wavefront per leaf, the leaf's particles up to 64 at a time.  With c particles in a
 // chunk, each takes g = floor(64 / c) lanes that split every tile (lane s of a group sweeps
 // slots s, s + g, ...), then a group reduction closes the particle: small leaves keep the
@@ -258,15 +266,19 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(MIXED && 
             }
             double dx, dy, dz;
             sep(k, dx, dy, dz);
-            // one root for q = r / h and 1 / (r + eps) = (1/r) (1 - eps / r), the next term of order
-            // (eps / r)^2; 2^-900 keeps the self pair (whose dx and D are zero) off zero
+            // one root for q = r / h and 1 / (r + eps) = (1/r) (1 - eps / r), whose next term (eps / r)^2 is
+            // below half an ulp for r >= 2^-25; nearer pairs (small units, or particles nearly at one
+            // place) take the reciprocal itself.  2^-1000 keeps the self pair, whose dx is zero, off zero
+            // and out of that branch
             double rij, rinv, V, G0, D;
-            sqrtAndInverse(dx * dx + dy * dy + dz * dz + 0x1p-900, rij, rinv);
+            sqrtAndInverse(dx * dx + dy * dy + dz * dz + 0x1p-1000, rij, rinv);
+            double r1 = fma(-kEps * rinv, rinv, rinv);
+            if (nearEps(rij)) r1 = recip(rij + kEps);
             const double q = fmin(rij * hinvi, kRad);
             kernVGD<double>(q, V, G0, D);
             rhoi += V;
             gradhi += G0;
-            const double rg = fma(-2.220446049250313e-16 * rinv, rinv, rinv) * (-kGp * D);
+            const double rg = r1 * (-kGp * D);
             const double rx = dx * rg * pmass, ry = dy * rg * pmass, rz = dz * rg * pmass;
             const double dvx = vxi - tj[3][k], dvy = vyi - tj[4][k], dvz = vzi - tj[5][k];
             divs += dvx * rx + dvy * ry + dvz * rz;

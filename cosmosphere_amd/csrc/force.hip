@@ -47,15 +47,6 @@ __global__ __launch_bounds__(256) void forcePrepKernel(const double* __restrict_
     divfac[i] = kCnormk * oinv * h4 / rho;
 }
 
-// 1/x for x > 0 by the hardware reciprocal and two Newton steps: within an ulp of the division,
-// at a third of its instructions.
-__device__ inline double recip(double x)
-{
-    double r = __builtin_amdgcn_rcp(x);
-    r = fma(r, fma(-x, r, 1.0), r);
-    return fma(r, fma(-x, r, 1.0), r);
-}
-
 // A double of lane p as a scalar (p wave-uniform).
 __device__ inline double laneD(double v, int p)
 {
