@@ -33,6 +33,7 @@ struct PassCtl
     unsigned long long nRem;            // particles in state != 0 at the start of the pass
     unsigned long long accIterating, accRem;   // ... of the next pass, summed by the compaction's blocks
     unsigned long long listNeed;        // list entries of the current pass
+    unsigned long long accList;         // ... summed by the scan's blocks (zero between scans)
     unsigned long long tBegin;          // wall clock at the start of the pass
     unsigned long long tStart, tEnd;    // density kernel span (wall clock) of the current pass
     unsigned long long listMean;        // list entries per active leaf of the last pass that built lists (0: none yet)

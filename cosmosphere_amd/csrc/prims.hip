@@ -34,8 +34,9 @@ constexpr int kScanTile    = kScanThreads * kScanItems;
 __device__ inline int scanCount(const PassCtl* ctl, int n) { return ctl ? min(n, (int)ctl->nAL) : n; }
 
 // LISTS: the offsets of a device-driven pass's lists.  The largest list's cost bucket goes to
-// listCtl->qBucket[0], and the last block to finish checks the total against the list buffer's
-// capacity: a pass that does not fit stops here with nothing changed.
+// ctl->qBucket[0], and the last block to finish checks the total against the list buffer's
+// capacity: a pass that does not fit stops here with nothing changed.  Totals are summed in 64 bits:
+// the offsets of lists of more than 2^32 entries wrap, and must not look as if they fitted.
 template<bool LISTS>
 __global__ __launch_bounds__(kScanThreads) void scanKernel(const uint32_t* __restrict__ in, uint32_t* __restrict__ out,
                                                            int n, ScanHead* __restrict__ head,
@@ -44,6 +45,7 @@ __global__ __launch_bounds__(kScanThreads) void scanKernel(const uint32_t* __res
                                                            PassCtl* __restrict__ ctl, unsigned long long cap)
 {
     __shared__ uint32_t waveTot[kScanThreads / kWave];
+    __shared__ unsigned long long waveTot64[kScanThreads / kWave];
     __shared__ uint32_t waveMax[kScanThreads / kWave];
     __shared__ uint32_t shTile, shEpoch, shBefore;
     if (ctl && ctl->skip) return;
@@ -60,18 +62,25 @@ __global__ __launch_bounds__(kScanThreads) void scanKernel(const uint32_t* __res
     const int base = tile * kScanTile + threadIdx.x * kScanItems;
     uint32_t v[kScanItems];
     uint32_t sum = 0, most = 0;
+    unsigned long long sum64 = 0;
 #pragma unroll
     for (int k = 0; k < kScanItems; ++k)
     {
         const int i = base + k;
         v[k] = (i < nEff) ? in[i] : 0u;
         sum += v[k];
+        sum64 += v[k];
         if constexpr (LISTS) most = max(most, v[k]);
     }
     // block-wide exclusive scan of the per-thread sums
     const uint32_t incl = waveInclusiveScan(sum);
     const int w = threadIdx.x / kWave;
     if (laneId() == kWave - 1) waveTot[w] = incl;
+    if (LISTS || total64)
+    {
+        sum64 = waveReduceSum(sum64);
+        if (laneId() == 0) waveTot64[w] = sum64;
+    }
     if constexpr (LISTS)
     {
         most = waveReduceMax(most);
@@ -100,9 +109,13 @@ __global__ __launch_bounds__(kScanThreads) void scanKernel(const uint32_t* __res
         run += v[k];
     }
     if (threadIdx.x != 0) return;
-    if (total64 && blockTot) atomicAdd(total64, (unsigned long long)blockTot);
+    unsigned long long blockTot64 = 0;
+    if (LISTS || total64)
+        for (int j = 0; j < kScanThreads / kWave; ++j) blockTot64 += waveTot64[j];
+    if (total64 && blockTot64) atomicAdd(total64, blockTot64);
     if constexpr (LISTS)
     {
+        if (tiles > 1 && blockTot64) atomicAdd(&ctl->accList, blockTot64);
         const uint32_t m = max(max(waveMax[0], waveMax[1]), max(waveMax[2], waveMax[3]));
         if (m > 1u) atomicMax(&ctl->qBucket[0], (uint32_t)listBucket(m));
         __threadfence();
@@ -116,7 +129,8 @@ __global__ __launch_bounds__(kScanThreads) void scanKernel(const uint32_t* __res
     }
     if constexpr (LISTS)
     {
-        const unsigned long long tot = tiles > 1 ? (uint32_t)published(words + tiles - 1) : blockTot;
+        const unsigned long long tot = tiles > 1 ? published(&ctl->accList) : blockTot64;
+        ctl->accList = 0ull;
         ctl->listNeed = tot;
         if (nEff > 0) ctl->listMean = tot / (unsigned long long)nEff;
         if (tot > cap)
