@@ -312,6 +312,7 @@ extern "C" void cosmo_ext_set_option(const char* name, double value)
     else if (nm == "list_heavy_factor") s.listHeavyFactor = std::max(0, (int)value);
     else if (nm == "grad_sym_lists") s.gradSymLists = (int)value;
     else if (nm == "split_len") s.splitLen = (int)value;
+    else if (nm == "split_parts") s.splitParts = std::max(0, (int)value);
     else if (nm == "sweep_split") s.sweepSplit = std::max(0, (int)value);
     else if (nm == "count_list") s.countList = (int)value;
     else if (nm == "list_expand_leaves") s.listExpandLeaves = (int)value;

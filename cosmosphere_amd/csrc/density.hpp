@@ -27,8 +27,9 @@ struct PassCtl
     uint32_t isNR;          // the current pass holds NR evaluations (else closures only)
     uint32_t qBucket[2];    // work queue: [0] largest cost bucket, [1] entries at its head (heavy items, split)
     uint32_t nSplit;        // items split over several wavefronts this pass
-    uint32_t nRange;        // ... mixed whole leaves asking for list ranges
-    uint32_t nParts;        // sub-items of the split items (slots of the partials asked for)
+    uint32_t nParts;        // sub-items of the split items (slots of the partials taken)
+    uint32_t nLong[168];    // whole-leaf items with more than kSplitLen list entries, by longBin
+    unsigned long long itemCosts;       // cost of all items of the pass (itemCost)
     unsigned long long nIterating;      // particles in state 1 at the start of the pass
     unsigned long long nRem;            // particles in state != 0 at the start of the pass
     unsigned long long accIterating, accRem;   // ... of the next pass, summed by the compaction's blocks
@@ -92,11 +93,13 @@ constexpr uint32_t kQueueStride = 32;
 // Split work items: sub-items run by different wavefronts, each summing a part of the item's pairs;
 // the last to finish adds the partial sums in sub-item order and ends the particles.  A part is a
 // range of the list or (mixed whole leaves, whose FP32 partials have to stay as they are) every
-// n-th of the tiles staged from the whole list.  Which items are split: loop.hip.
+// n-th of the tiles staged from the whole list.  Which items are split: loop.hip; the sub-items of
+// a pass always fit their slots (an item cut or not as the slots last would be cut in one run of a solve
+// and not in the next, and its sums rounded otherwise).
 constexpr int kSplitLen = 2048;         // mixed whole leaves: list ranges beyond this many entries ...
 constexpr int kMaxSplit = 256;          // ... of at most this many items a pass
 constexpr int kMaxSub   = 32;           // sub-items of an item
-constexpr int kMaxParts = 16384;        // sub-items of a pass's split items
+constexpr int kMaxParts = 32768;        // sub-items of a pass's split items
 
 // A queue-head entry's sub-item: its number, count, kind and the item's first slot of the partials.
 constexpr uint32_t kSubTiles = 1u << 12;
@@ -108,8 +111,25 @@ __device__ inline uint32_t subNumber(uint32_t s) { return s & 63u; }
 __device__ inline uint32_t subCount(uint32_t s) { return (s >> 6) & 63u; }
 __device__ inline uint32_t subPart0(uint32_t s) { return s >> 16; }
 
+// What an item costs: its list entries, each staged (as much work as kStageCost particles' pairs
+// with it) and swept for the particles evaluated.
+constexpr uint32_t kStageCost = 8;
+__device__ inline uint32_t itemCost(uint32_t len, uint32_t particles)
+{
+    return (uint32_t)min((unsigned long long)len * (kStageCost + particles), 0x7FFFFFFFull);
+}
+
 // Cost bucket of a list of len entries: floor(log2).
 __device__ inline int listBucket(uint32_t len) { return 31 - __clz((int)(len | 1u)); }
+
+// Finer ones of lists of at least kSplitLen = 2^11 entries: eight to a power of two.
+constexpr int kLongBins = (32 - 11) * 8;
+static_assert(kSplitLen == 1 << 11 && kLongBins == sizeof(PassCtl::nLong) / sizeof(uint32_t), "longBin");
+__device__ inline int longBin(uint32_t len)
+{
+    const int b = listBucket(len);
+    return (b - 11) * 8 + (int)((len >> (b - 3)) & 7u);
+}
 
 // Work items of an active leaf with `remaining` particles still to evaluate.
 __device__ inline uint32_t itemsOf(uint32_t remaining, int sparse)

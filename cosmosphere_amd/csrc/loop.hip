@@ -72,15 +72,8 @@ struct ItemArgs
     int             splitLen;   // list length beyond which heavy items are split, 0: none are; < 0: by the pass's load
     int             waves;      // of the density kernel's grid
     int             mixed;
+    int             maxParts;   // slots of the sub-items' partials
 };
-
-// What an item costs: its list entries, each staged (as much work as kStageCost particles' pairs
-// with it) and swept for the particles evaluated.
-constexpr uint32_t kStageCost = 8;
-__device__ inline uint32_t itemCost(uint32_t len, uint32_t particles)
-{
-    return (uint32_t)min((unsigned long long)len * (kStageCost + particles), 0x7FFFFFFFull);
-}
 
 // What makes an item of a pass heavy.
 struct QueueRule
@@ -89,6 +82,8 @@ struct QueueRule
     unsigned long long heavyLen;   // ... with at least this many entries,
     uint32_t           cost;       // or a cost above this;
     uint32_t           part;       // the cost of a sub-item
+    int                range;      // mixed whole leaves: list ranges for lists in this longBin or above
+    uint32_t           rangeLen;   // list entries of a sub-item that is a range by length
 };
 
 // Work queue: the heavy items first (qOrder[0, qBucket[1]), in no particular order: started last
@@ -121,11 +116,11 @@ __device__ inline void queueItem(const ItemArgs& A, const QueueRule& R, bool is,
         want = 1u;
         if (A.splitLen > 0)
         {
-            if (batch && longest && len > (uint32_t)A.splitLen) want = (len + (uint32_t)A.splitLen - 1u) / (uint32_t)A.splitLen;
+            if (batch && longest && len > R.rangeLen) want = (len + R.rangeLen - 1u) / R.rangeLen;
         }
         else if (A.splitLen < 0 && batch)
         {
-            range = A.mixed && !onePart && longest && len > (uint32_t)kSplitLen;
+            range = A.mixed && !onePart && longest && len > (uint32_t)kSplitLen && longBin(len) >= R.range;
             if (range) want = (len + (uint32_t)kSplitLen - 1u) / (uint32_t)kSplitLen;
             else       want = min((cost + R.part - 1u) / R.part, max(len / kMinPart, 1u));
             if (A.mixed && !onePart && !range)
@@ -141,14 +136,6 @@ __device__ inline void queueItem(const ItemArgs& A, const QueueRule& R, bool is,
         if (is) A.qFlag[k] = 0;
         return;
     }
-    if (A.mixed && ballot64(range))
-    {
-        const uint64_t m = ballot64(range);
-        uint32_t s = 0;
-        if (laneId() == 0) s = atomicAdd(&C->nRange, (uint32_t)__popcll(m));
-        s = __builtin_amdgcn_readfirstlane(s) + (uint32_t)__popcll(m & lanemaskLt());
-        if (range && s >= (uint32_t)kMaxSplit) want = 1u;
-    }
     uint32_t part0 = 0u;
     if (ballot64(want > 1u))
     {
@@ -156,7 +143,7 @@ __device__ inline void queueItem(const ItemArgs& A, const QueueRule& R, bool is,
         uint32_t p = 0;
         if (laneId() == kWave - 1) p = atomicAdd(&C->nParts, incl);
         part0 = (uint32_t)__shfl((int)p, kWave - 1, kWave) + incl - parts;
-        if (part0 + parts > (uint32_t)kMaxParts) want = min(want, 1u);
+        if (part0 + parts > (uint32_t)A.maxParts) want = min(want, 1u);   // (never: QueueRule)
         const uint64_t m = ballot64(want > 1u);
         if (laneId() == 0 && m) atomicAdd(&C->nSplit, (uint32_t)__popcll(m));
     }
@@ -188,14 +175,41 @@ __global__ __launch_bounds__(kItemThreads) void itemsKernel(ItemArgs A)
     // well above the mean
     R.heavyLen = (int)C->nItems <= kFewItems ? 0ull : kHeavyMean * mean;
     R.cost = R.part = 0x7FFFFFFFu;
+    R.range = kLongBins;
+    R.rangeLen = (uint32_t)max(A.splitLen, 1);
+    // An item cut into parts of cost p has fewer than 2 cost / p of them (one with a single part is not
+    // cut): with p at least 2 / slots of the cost of all items, the slots are enough whatever the items are.
+    // Which ones are cut then does not depend on the order in which wavefronts get here.
+    const unsigned long long costs = C->itemCosts;
+    if (A.splitLen > 0)
+    {
+        const unsigned long long entries = costs / (kStageCost + 1u);   // at least those of all items' lists
+        R.rangeLen = (uint32_t)min(max((unsigned long long)R.rangeLen, 2ull * entries / (unsigned long long)A.maxParts + 1ull),
+                                   0x7FFFFFFFull);
+    }
     if (A.splitLen < 0)
     {
+        // list ranges of the longest lists, by whole bins, up to kMaxSplit items: lane l counts the l-th bin
+        // from the longest list's bucket down (kHeavySpan + 1 buckets: all that can be heavy)
+        int slots = A.maxParts;
+        if (A.mixed)
+        {
+            const uint32_t most = (uint32_t)min(kMaxSplit, A.maxParts / (2 * kMaxSub));
+            const uint32_t least = (uint32_t)min(max(R.heavyLen, (unsigned long long)kSplitLen), 0xFFFFFFFFull);
+            const int bin = ((int)C->qBucket[0] - 11) * 8 + 7 - laneId();
+            const bool in = laneId() < (kHeavySpan + 1) * 8 && bin >= longBin(least);
+            const uint32_t above = waveInclusiveScan(in ? C->nLong[bin] : 0u);
+            const uint64_t fit = ballot64(in && above <= most);   // a run of lanes from 0 on
+            if (fit) R.range = ((int)C->qBucket[0] - 11) * 8 + 8 - __popcll(fit);
+            slots -= (int)most * kMaxSub;
+        }
+        const unsigned long long leastPart = 2ull * costs / (unsigned long long)slots + 1ull;
         // mean cost of the pass's items and the share of one of the grid's wavefronts
         const double mc = C->perParticle ? (double)itemCost((uint32_t)mean, 1u)
                                          : (double)mean * ((double)kStageCost + (double)C->nRem / (double)max(n, 1));
         const double share = mc * (double)C->nItems / (double)max(A.waves, 1);
         R.cost = (uint32_t)fmin(fmax(share / kHeadDiv, fmin(kHeadMean * mc, share / 2)), 2e9);
-        R.part = (uint32_t)fmin(fmax(share / 2, 8.0), 2e9);
+        R.part = (uint32_t)min(max((unsigned long long)fmin(fmax(share / 2, 8.0), 2e9), leastPart), 0x7FFFFFFFull);
     }
     if (!C->perParticle)
     {
@@ -406,6 +420,7 @@ __global__ __launch_bounds__(kCompactThreads) void compactKernel(CompactArgs A)
     }
     if (t < 2) A.heavyN[t] = 0;
     if (t < (int)kQueueHeads) A.qHead[t * kQueueStride] = 0u;
+    if (t < kLongBins) C->nLong[t] = 0u;
     __syncthreads();
     if (t != 0) return;
     __threadfence();
@@ -464,8 +479,8 @@ __global__ __launch_bounds__(kCompactThreads) void compactKernel(CompactArgs A)
     C->qBucket[0] = 0u;
     C->qBucket[1] = 0u;
     C->nSplit = 0u;
-    C->nRange = 0u;
     C->nParts = 0u;
+    C->itemCosts = 0ull;
     C->tStart = ~0ull;
     C->tEnd = 0ull;
     C->tBegin = clockNow();
@@ -518,7 +533,7 @@ void enqueuePass(State& s, const Plan& P)
 {
     hipStream_t st = s.stream;
     launchGatherListsDevice(s, P.items.leaves, P.L, P.jc, nullptr, nullptr, P.ctl);
-    scanLists(P.jc, P.jo, P.L, P.scan, P.ctl, P.listCap, st);
+    scanLists(P.jc, P.jo, P.L, P.scan, P.ctl, P.listCap, st, P.items.leafRem, P.items.sparse);
     launchGatherListsDevice(s, P.items.leaves, P.L, P.jc, P.jo, P.jList, P.ctl);
     if (P.listCand)
         launchListCand(P.ctl, P.L, P.items.leaves, P.jo, P.jc, P.jList, P.items.layout, P.items.state, P.listCand, st);
@@ -643,6 +658,7 @@ int deviceLoop(State& s, const DeviceLoopArgs& in, Timings& t)
     int* qOrder = s.qOrder.get<int>(qCap);
     uint8_t* qFlag = s.qFlag.get<uint8_t>(qCap);
     uint32_t* qSub = s.splitLen != 0 ? s.qSub.get<uint32_t>(qCap) : nullptr;
+    P.items.maxParts = s.splitParts > 0 ? std::min(s.splitParts, kMaxParts) : kMaxParts;
     double* splitPart = s.splitPart.get<double>((size_t)kMaxParts * kWave * 2);
     uint32_t* splitDone = s.splitDone.get<uint32_t>((size_t)kMaxParts);
     fillU32(splitDone, 0u, (size_t)kMaxParts, st);   // every pass leaves them at 0
@@ -829,6 +845,8 @@ int deviceLoop(State& s, const DeviceLoopArgs& in, Timings& t)
             hc.overflow = 0u;
             hc.skip = 0u;
             hc.qBucket[0] = 0u;
+            hc.itemCosts = 0ull;
+            std::memset(hc.nLong, 0, sizeof(hc.nLong));
             HIP_CHECK(hipMemcpyAsync(P.ctl, &hc, sizeof(hc), hipMemcpyHostToDevice, st));
             fillU32(reinterpret_cast<uint32_t*>(heavyN), 0u, 2, st);   // the count walk runs again
             if (s.useGraph) capture();

@@ -42,8 +42,11 @@ __global__ __launch_bounds__(kScanThreads) void scanKernel(const uint32_t* __res
                                                            int n, ScanHead* __restrict__ head,
                                                            unsigned long long* __restrict__ words,
                                                            unsigned long long* __restrict__ total64,
-                                                           PassCtl* __restrict__ ctl, unsigned long long cap)
+                                                           PassCtl* __restrict__ ctl, unsigned long long cap,
+                                                           const uint32_t* __restrict__ leafRem, int sparse)
 {
+    __shared__ uint32_t longLists[LISTS ? kLongBins : 1];
+    __shared__ unsigned long long waveCost[LISTS ? kScanThreads / kWave : 1];
     __shared__ uint32_t waveTot[kScanThreads / kWave];
     __shared__ unsigned long long waveTot64[kScanThreads / kWave];
     __shared__ uint32_t waveMax[kScanThreads / kWave];
@@ -57,12 +60,14 @@ __global__ __launch_bounds__(kScanThreads) void scanKernel(const uint32_t* __res
         shTile = tiles > 1 ? atomicAdd(&head->ticket, 1u) : 0u;
         shEpoch = head->epoch;
     }
+    if constexpr (LISTS)
+        if (threadIdx.x < kLongBins) longLists[threadIdx.x] = 0u;
     __syncthreads();
     const int tile = (int)shTile;
     const int base = tile * kScanTile + threadIdx.x * kScanItems;
     uint32_t v[kScanItems];
     uint32_t sum = 0, most = 0;
-    unsigned long long sum64 = 0;
+    unsigned long long sum64 = 0, cost = 0;
 #pragma unroll
     for (int k = 0; k < kScanItems; ++k)
     {
@@ -70,7 +75,17 @@ __global__ __launch_bounds__(kScanThreads) void scanKernel(const uint32_t* __res
         v[k] = (i < nEff) ? in[i] : 0u;
         sum += v[k];
         sum64 += v[k];
-        if constexpr (LISTS) most = max(most, v[k]);
+        if constexpr (LISTS)
+        {
+            most = max(most, v[k]);
+            if (leafRem && i < nEff)
+            {
+                const uint32_t rem = leafRem[i];
+                const bool parts = ctl->perParticle && rem <= (uint32_t)sparse;   // an item for each particle
+                cost += parts ? (unsigned long long)rem * itemCost(v[k], 1u) : (unsigned long long)itemCost(v[k], rem);
+                if (!parts && v[k] > (uint32_t)kSplitLen) atomicAdd(&longLists[longBin(v[k])], 1u);
+            }
+        }
     }
     // block-wide exclusive scan of the per-thread sums
     const uint32_t incl = waveInclusiveScan(sum);
@@ -84,7 +99,12 @@ __global__ __launch_bounds__(kScanThreads) void scanKernel(const uint32_t* __res
     if constexpr (LISTS)
     {
         most = waveReduceMax(most);
-        if (laneId() == 0) waveMax[w] = most;
+        cost = waveReduceSum(cost);
+        if (laneId() == 0)
+        {
+            waveMax[w] = most;
+            waveCost[w] = cost;
+        }
     }
     __syncthreads();
     uint32_t waveOff = 0, blockTot = 0;
@@ -108,6 +128,8 @@ __global__ __launch_bounds__(kScanThreads) void scanKernel(const uint32_t* __res
         if (i <= nEff) out[i] = run;   // out[nEff]: the total
         run += v[k];
     }
+    if constexpr (LISTS)
+        if (threadIdx.x < kLongBins && longLists[threadIdx.x]) atomicAdd(&ctl->nLong[threadIdx.x], longLists[threadIdx.x]);
     if (threadIdx.x != 0) return;
     unsigned long long blockTot64 = 0;
     if (LISTS || total64)
@@ -115,6 +137,8 @@ __global__ __launch_bounds__(kScanThreads) void scanKernel(const uint32_t* __res
     if (total64 && blockTot64) atomicAdd(total64, blockTot64);
     if constexpr (LISTS)
     {
+        const unsigned long long c = waveCost[0] + waveCost[1] + waveCost[2] + waveCost[3];
+        if (c) atomicAdd(&ctl->itemCosts, c);
         if (tiles > 1 && blockTot64) atomicAdd(&ctl->accList, blockTot64);
         const uint32_t m = max(max(waveMax[0], waveMax[1]), max(waveMax[2], waveMax[3]));
         if (m > 1u) atomicMax(&ctl->qBucket[0], (uint32_t)listBucket(m));
@@ -161,16 +185,16 @@ void scanExclusive(const uint32_t* in, uint32_t* out, int n, DevBuf& scratch, un
     char* sc = scanReserve(scratch, n, st);
     scanKernel<false><<<(int)scanTiles(n), kScanThreads, 0, st>>>(
         in, out, n, reinterpret_cast<ScanHead*>(sc), reinterpret_cast<unsigned long long*>(sc + sizeof(ScanHead)), total64,
-        nullptr, 0ull);
+        nullptr, 0ull, nullptr, 0);
     LAUNCH_CHECK();
 }
 
 void scanLists(const uint32_t* counts, uint32_t* offsets, int n, char* scratch, PassCtl* ctl, unsigned long long cap,
-               hipStream_t st)
+               hipStream_t st, const uint32_t* leafRem, int sparse)
 {
     scanKernel<true><<<(int)scanTiles(n), kScanThreads, 0, st>>>(
         counts, offsets, n, reinterpret_cast<ScanHead*>(scratch),
-        reinterpret_cast<unsigned long long*>(scratch + sizeof(ScanHead)), nullptr, ctl, cap);
+        reinterpret_cast<unsigned long long*>(scratch + sizeof(ScanHead)), nullptr, ctl, cap, leafRem, sparse);
     LAUNCH_CHECK();
 }
 

@@ -27,10 +27,11 @@ void scanExclusive(const uint32_t* in, uint32_t* out, int n, DevBuf& scratch, un
                    hipStream_t st);
 
 // Device-driven pass: the offsets of the ctl->nAL lists from their counts (n: their capacity),
-// the longest list's cost bucket, and the check of the total against cap entries (prims.hip).
+// the longest list's cost bucket, and the check of the total against cap entries (prims.hip); with
+// the lists' particles still to evaluate in leafRem also the cost of the pass's items and its long lists.
 // Nothing when ctl->skip.  scratch: scanReserve'd for n before the capture.
 void scanLists(const uint32_t* counts, uint32_t* offsets, int n, char* scratch, PassCtl* ctl, unsigned long long cap,
-               hipStream_t st);
+               hipStream_t st, const uint32_t* leafRem = nullptr, int sparse = 0);
 
 // Stable ascending sort of (keys, vals) by the 8-bit digits that hold a bit of `varying`; the
 // other digits must be shared by all keys, or in order already among keys that the sorted digits

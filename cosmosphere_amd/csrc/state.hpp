@@ -217,6 +217,7 @@ struct State
     double listMeanGather = 0.0;   // entries per leaf of the last all-leaf gather / symmetric list build
     double listMeanSym = 0.0;
     int listExpandLeaves = -1;     // verification: block walk expands nodes above this many leaves (-1: default)
+    int splitParts = 0;            // verification: sub-items of a pass at most (0: kMaxParts)
     int splitLen = -1;             // device-driven loop: heavy items with longer lists are split (-1: default, 0: off)
     int forceRounds = 1;           // mixed force pass: 1 shares each tile's accepted pairs over the lanes, 0 lanes keep their own slots
     int countList = 0;             // count the list candidates of each pass (a separate kernel; for reports), over the reference's untrimmed lists

@@ -119,7 +119,8 @@ int cosmo_ext_solve_dens_h(int n, double pmass, int mode, int withGradients, int
  * more leaves than this are expanded into separate walks, default 256), "list_slot" (verification:
  * tokens kept per list between its count and its fill, at most; default 0: by the number of leaves),
  * "split_len" (device-driven loop: a heavy work item whose list has more entries is split over several
- * wavefronts; 0: never; default -1: items are split by the pass's load), "sweep_split" (gradient
+ * wavefronts; 0: never; default -1: items are split by the pass's load), "split_parts" (verification:
+ * sub-items of a pass's split items, at most; default 0: 32768), "sweep_split" (gradient
  * sweep and force pass: the particles of a leaf whose list has more entries go one per wavefront,
  * default 512; 0: never), "list_heavy_factor" (a walk also goes to the block walk past this many times the previous build's typical walk,
  * default 8; 0: the launch-size rule only), "tile_depth" (device-driven loop: j-slots per LDS
