@@ -47,7 +47,8 @@ __global__ __launch_bounds__(256) void forcePrepKernel(const double* __restrict_
     divfac[i] = kCnormk * oinv * h4 / rho;
 }
 
-// A double of lane p as a scalar (p wave-uniform).
+// A double of lane p as a scalar (p wave-uniform).  With every lane active: a register that was spilled
+// or recomputed under divergence holds nothing for the lanes that were off.
 __device__ inline double laneD(double v, int p)
 {
     const long long x = __double_as_longlong(v);
@@ -150,14 +151,26 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(PER ? 1 :
             auto keep = [&](int jl) {
                 double hj = A.hmaxLeaf[jl];
                 const double rj = (isfinite(hj) && hj > 0.0) ? kRad * hj : 0.0;
+                // open: the chunk's particles from their owner lanes, read anew for 64 entries; no lane
+                // leaves the loop before the last one may, so that every owner lane is active
+                uint32_t own = ic;
+                asm volatile("" : "+v"(own));
+                double kx = 0, ky = 0, kz = 0, kr = 0;
+                if constexpr (!PER)
+                {
+                    kx = A.x[own]; ky = A.y[own]; kz = A.z[own];
+                    kr = kRad * A.h[own];
+                }
+                bool hit = false;
                 for (int k = 0; k < c; ++k)
                 {
-                    const double px = PER ? cp[0][k] : laneD(xc, k), py = PER ? cp[1][k] : laneD(yc, k);
-                    const double pz = PER ? cp[2][k] : laneD(zc, k), pr = PER ? cp[3][k] : laneD(rc, k);
+                    const double px = PER ? cp[0][k] : laneD(kx, k), py = PER ? cp[1][k] : laneD(ky, k);
+                    const double pz = PER ? cp[2][k] : laneD(kz, k), pr = PER ? cp[3][k] : laneD(kr, k);
                     const double r = fmax(pr, rj);
-                    if (pointLeafGap2<PER>(px, py, pz, A.lbox, A.lboxN, jl, box) <= r * r * kCullSlack) return true;
+                    hit |= pointLeafGap2<PER>(px, py, pz, A.lbox, A.lboxN, jl, box) <= r * r * kCullSlack;
+                    if (!ballot64(!hit)) break;
                 }
-                return false;
+                return hit;
             };
             auto keepJ = [&](int j) {
                 const double r = fmax(rChunk, kRad * A.h[j]);
@@ -682,14 +695,15 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(4))) void
             auto keep = [&](int jl) {
                 double hj = A.hmaxLeaf[jl];
                 const double rj = (isfinite(hj) && hj > 0.0) ? kRad * hj : 0.0;
-                for (int k = 0; k < c; ++k)
+                bool hit = false;
+                for (int k = 0; k < c; ++k)   // (no lane leaves before the last one may: laneD)
                 {
                     const double r = fmax(laneD(rhi, k), rj);
-                    if (pointLeafGap2<PER>(laneD(xi, k), laneD(yi, k), laneD(zi, k), A.lbox, A.lboxN, jl, box) <=
-                        r * r * kCullSlack)
-                        return true;
+                    hit |= pointLeafGap2<PER>(laneD(xi, k), laneD(yi, k), laneD(zi, k), A.lbox, A.lboxN, jl, box) <=
+                           r * r * kCullSlack;
+                    if (!ballot64(!hit)) break;
                 }
-                return false;
+                return hit;
             };
             auto keepJ = [&](int j) {
                 const double cc[3] = {cbox[0], cbox[1], cbox[2]};

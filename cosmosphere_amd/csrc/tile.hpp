@@ -88,7 +88,9 @@ __device__ inline void forEachTileIf(int* __restrict__ segStart, int* __restrict
 // and which keepJ(j) accepts, as full 64-slot tiles: each round every lane tests one candidate,
 // the accepted ones join a queue (LDS, 2 kWave entries), and each time 64 are queued (and once
 // more for the rest at the end) load(slot, j) runs for every slot, then consume(nt).  A
-// particle-level test that rejects most of a leaf's particles then costs no pair sweeps.
+// particle-level test that rejects most of a leaf's particles then costs no pair sweeps.  keep(jl) runs
+// with every lane active (it may read other lanes' registers); lanes past the list's end repeat its
+// last entry.
 template<class Keep, class KeepJ, class Load, class Consume>
 __device__ inline void forEachTileCompact(int* __restrict__ segStart, int* __restrict__ segJ, int* __restrict__ head,
                                           int* __restrict__ queue,
@@ -102,14 +104,12 @@ __device__ inline void forEachTileCompact(int* __restrict__ segStart, int* __res
     {
         const uint32_t e = e0 + lane;
         int js = 0, jc = 0;
-        if (e < hi)
+        const int jl = jList[min(e, hi - 1u)];
+        const bool kept = keep(jl);
+        if (kept && e < hi)
         {
-            const int jl = jList[e];
-            if (keep(jl))
-            {
-                js = (int)layout[jl];
-                jc = (int)layout[jl + 1] - js;
-            }
+            js = (int)layout[jl];
+            jc = (int)layout[jl + 1] - js;
         }
         const int incl  = waveInclusiveScan(jc);
         const int total = lastLane(incl);   // wave-uniform
