@@ -307,6 +307,13 @@ extern "C" void cosmo_ext_set_option(const char* name, double value)
     else if (nm == "units") s.units = (int)value;
     else if (nm == "loop_blocks_scale") s.loopBlockScale = std::max(1, (int)value);
     else if (nm == "loop_list_cap") s.loopListCap = (long long)value;
+    else if (nm == "alloc_limit")
+    {
+        s.allocLimit = (size_t)std::max(0.0, value);
+        s.slotFor = -1;
+        if (s.slotTok.p) HIP_CHECK(hipFree(s.slotTok.p));
+        s.slotTok = DevBuf();
+    }
     else if (nm == "list_slot") s.listSlot = std::max(0, (int)value);
     else if (nm == "list_heavy_steps") s.listHeavySteps = (int)value;
     else if (nm == "list_heavy_factor") s.listHeavyFactor = std::max(0, (int)value);
@@ -379,6 +386,7 @@ extern "C" double cosmo_ext_get_stat(const char* name)
     if (nm == "graph_captures") return t.graphCaptures;
     if (nm == "loop") return s.loopMode;
     if (nm == "bucket") return s.bucket;
+    if (nm == "list_slot_tokens") return s.slotCap;
     if (nm.compare(0, 5, "tune_") == 0) return tuneStat(nm);
     if (nm == "graph") return s.useGraph;
     if (nm == "graph_passes") return s.graphPasses;

@@ -229,7 +229,7 @@ struct ListArgs
     const int*      fullStart;    // the full-walk order (buildTree): per node, its start; nullptr: off
     const int*      fullOrder;    // ... per position, the leaf
     int*            slotTok;      // light lists: the count walk's tokens, slotCap per position
-    int             slotCap;      // ... (listSlotTokens)
+    int             slotCap;      // ... (reserveListSlots)
                                   // (>= 0: a leaf; < 0: ~C, a node whose whole subtree is listed)
     uint32_t*       slotN;        // ... per position: their number, ~0u if not kept (the fill walks)
 };
@@ -841,6 +841,24 @@ static void launchList(const ListArgs& a, bool periodic, hipStream_t st)
     LAUNCH_CHECK();
 }
 
+void reserveListSlots(State& s)
+{
+    if (s.slotFor == s.leafCap) return;
+    int n = listSlotTokens(s.leafCap);
+    auto bytes = [&]() { return ((size_t)s.leafCap + 1) * (size_t)n * sizeof(int); };
+    if (n > kListSlotTok && bytes() > s.slotTok.cap)
+    {
+        size_t freeBytes = 0, total = 0;
+        HIP_CHECK(hipMemGetInfo(&freeBytes, &total));
+        freeBytes += s.slotTok.cap;   // given back if the buffer grows
+        while (n > kListSlotTok && bytes() > freeBytes / 16) n /= 2;
+        while (n > kListSlotTok && !s.slotTok.tryReserve(bytes(), s.allocLimit)) n /= 2;
+    }
+    s.slotTok.reserve(bytes());
+    s.slotCap = n;
+    s.slotFor = s.leafCap;
+}
+
 static ListArgs listArgs(State& s, const int* leaves, int nLeaves, bool symmetric, bool tight)
 {
     ListArgs a;
@@ -867,8 +885,9 @@ static ListArgs listArgs(State& s, const int* leaves, int nLeaves, bool symmetri
     a.fullStart = s.fullStart.as<int>();
     a.fullOrder = s.fullStart.p ? s.fullOrder.as<int>() : nullptr;
     a.tokAt = s.tokAt.get<uint2>((size_t)s.leafCap + 1);
-    a.slotCap = s.listSlot > 0 ? std::min(s.listSlot, listSlotTokens(s.leafCap)) : listSlotTokens(s.leafCap);
-    a.slotTok = s.slotTok.get<int>(((size_t)s.leafCap + 1) * listSlotTokens(s.leafCap));
+    reserveListSlots(s);
+    a.slotCap = s.listSlot > 0 ? std::min(s.listSlot, s.slotCap) : s.slotCap;
+    a.slotTok = s.slotTok.as<int>();
     a.slotN = s.slotN.get<uint32_t>((size_t)s.leafCap + 1);
     a.heavySteps = s.listHeavySteps > 0 ? s.listHeavySteps : kHeavySteps;
     a.expandLeaves = s.listExpandLeaves >= 0 ? s.listExpandLeaves : kExpandLeaves;

@@ -562,7 +562,7 @@ std::vector<unsigned long long> planKey(const State& s, const Plan& P, int K)
     k.push_back((unsigned long long)s.nSets);
     k.push_back((unsigned long long)s.nodeCap);
     k.push_back((unsigned long long)s.leafCap);
-    for (int v : {s.listSlot, s.listHeavySteps, s.listHeavyFactor, s.listExpandLeaves, s.countList ? 1 : 0})   // of the list walks
+    for (int v : {s.slotCap, s.listSlot, s.listHeavySteps, s.listHeavyFactor, s.listExpandLeaves, s.countList ? 1 : 0})   // of the list walks
         k.push_back((unsigned long long)(long long)v);
     k.push_back((unsigned long long)K);
     return k;
@@ -675,7 +675,7 @@ int deviceLoop(State& s, const DeviceLoopArgs& in, Timings& t)
     s.heavyFlag.get<uint8_t>((size_t)L + 1);
     s.tokPool.get<int2>((size_t)kListTokPool);
     s.tokAt.get<uint2>((size_t)L + 1);
-    s.slotTok.get<int>(((size_t)L + 1) * listSlotTokens(L));
+    reserveListSlots(s);
     s.slotN.get<uint32_t>((size_t)L + 1);
     const int instance = s.precision | (in.periodic ? 2 : 0) | (in.da.cull ? 4 : 0) | in.da.tileDepth << 3;
     if (s.loopBlocksFor != instance)

@@ -36,6 +36,25 @@ struct DevBuf
         HIP_CHECK(hipMalloc(&p, want));
         cap = want;
     }
+    // reserve(), but false (and an empty buffer) where the memory is not there, or beyond
+    // tryLimit (verification; 0: none).
+    bool tryReserve(size_t bytes, size_t tryLimit)
+    {
+        if (bytes <= cap) return true;
+        if (p) HIP_CHECK(hipFree(p));
+        p = nullptr;
+        cap = 0;
+        const size_t want = bytes + bytes / 8 + 256;
+        if (tryLimit && want > tryLimit) return false;
+        if (hipMalloc(&p, want) != hipSuccess)
+        {
+            (void)hipGetLastError();
+            p = nullptr;
+            return false;
+        }
+        cap = want;
+        return true;
+    }
     template<class T> T* as() const { return static_cast<T*>(p); }
     template<class T> T* get(size_t n) { reserve(n * sizeof(T)); return as<T>(); }
 };
@@ -170,7 +189,8 @@ struct State
     DevBuf itemCount, itemCountAlt, itemOff, itemPos, itemPart;   // NR work items
     DevBuf jCount, jOffset, jList;
     DevBuf heavyList, heavyFlag, heavyN;   // lists walked by a whole block (long walks)
-    DevBuf slotTok, slotN;                 // light lists: the count walk's tokens (listSlotTokens per position) and their number
+    DevBuf slotTok, slotN;                 // light lists: the count walk's tokens (slotCap per position) and their number
+    int    slotCap = 0, slotFor = -1;      // ... tokens per position, and the leafCap they are reserved for (reserveListSlots)
     DevBuf tokPool, tokAt;                 // ... their tokens, kept by the count pass for the fill
     DevBuf qSub, splitPart, splitDone;     // device-driven loop: heavy items split over wavefronts
     DevBuf sweepFlag, sweepCount, sweepOff, sweepItems;   // gradient / force sweeps: per-particle items of long lists
@@ -210,6 +230,7 @@ struct State
     int      loopBlockScale = 4;   // persistent density grid: resident blocks x scale / 4
     int      loopBlocks = 0, loopBlocksFor = -1;   // ... and the kernel instance they are counted for
     long long loopListCap = 0;     // verification: starting list capacity of the device-driven loop (0: auto)
+    size_t allocLimit = 0;         // verification: optional buffers larger than this are taken to be refused (0: none)
     int listSlot = 0;              // verification: tokens the count walk keeps per list, at most (0: listSlotTokens)
     int listHeavySteps = 0;        // verification: walk steps before a list goes to the block walk (0: default)
     int gradSymLists = 1;          // gradient sweep over the symmetric lists, which the force pass reuses

@@ -29,6 +29,12 @@ inline int listSlotTokens(int leafCap)
     return n;
 }
 
+// The slots of the present leafCap: s.slotTok, and their length in s.slotCap.  More than the least length
+// is taken only out of a sixteenth of the card's free memory, and where the allocation succeeds: it
+// saves time, and must not fail a solve, or a later allocation, that fits without it.  Called before
+// any capture.
+void reserveListSlots(State& s);
+
 // Box, keys, sort, permutation (x, y, z, h and, if withVelAcc, v and a), leaf tree, node
 // geometry, layout and particle -> leaf map for the sets described in s.
 // periodicBox: nullptr (open, fitted boxes) or 6 doubles per set.

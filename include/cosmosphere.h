@@ -118,6 +118,7 @@ int cosmo_ext_solve_dens_h(int n, double pmass, int mode, int withGradients, int
  * walk steps per 32768 lists before a list is handed to a whole block, default 256; nodes with
  * more leaves than this are expanded into separate walks, default 256), "list_slot" (verification:
  * tokens kept per list between its count and its fill, at most; default 0: by the number of leaves),
+ * "alloc_limit" (verification: optional buffers of more bytes are taken to be refused; 0: none),
  * "split_len" (device-driven loop: a heavy work item whose list has more entries is split over several
  * wavefronts; 0: never; default -1: items are split by the pass's load), "split_parts" (verification:
  * sub-items of a pass's split items, at most; default 0: 32768), "sweep_split" (gradient
