@@ -583,8 +583,9 @@ std::string signatureOf(const char* kind, const State& s, int n, int periodic, d
         }
     char b[256];
     std::snprintf(b, sizeof(b), "%s n=%d sets=%zu sizes=%016llx R=%g precision=%d periodic=%d tolh=%g hfact=%g "
-                                "closure=%d max_iter=%d",
-                  kind, n, counts.size(), h, kRad, s.precision, periodic, tolh, hfact, s.closureOn, s.maxIter);
+                                "closure=%d max_iter=%d kernels=%d",
+                  kind, n, counts.size(), h, kRad, s.precision, periodic, tolh, hfact, s.closureOn, s.maxIter,
+                  kTuneKernels);
     return b;
 }
 } // namespace

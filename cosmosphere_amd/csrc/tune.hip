@@ -84,7 +84,8 @@ std::map<std::string, TuneParams>& memo()
     return *m;
 }
 
-// COSMO_TUNE_CACHE: one line per signature, "signature<TAB>options".
+// COSMO_TUNE_CACHE: one line per signature, "signature<TAB>options" (lines of other builds' kernels, by the
+// signature's kTuneKernels, match no workload and stay as they are).
 void loadFileCache()
 {
     static bool loaded = false;

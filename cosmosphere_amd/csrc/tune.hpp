@@ -28,6 +28,12 @@ struct TuneParams
     int tileDepth;     // device loop: j-slots per LDS tile of whole-leaf items (64 or 128)
 };
 
+// Part of a workload's signature, so that choices kept in a file (COSMO_TUNE_CACHE) by a build whose
+// kernels the options meant something else to are not taken: raised with the density grid, queue or
+// tiles.  1 (lines without it): persistent grid of the 64-slot instance; 2: of the launched one, queue
+// over 32 counters, items cut by the pass's load.
+constexpr int kTuneKernels = 2;
+
 TuneParams currentParams(const State& s);
 void       applyParams(State& s, const TuneParams& p);
 std::string describe(const TuneParams& p);
