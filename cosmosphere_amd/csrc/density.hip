@@ -24,7 +24,6 @@
 namespace csph
 {
 
-
 __global__ void initActiveKernel(uint8_t* __restrict__ active, int nAlive, int n, double* __restrict__ rho,
                                  double* __restrict__ gradh)
 {

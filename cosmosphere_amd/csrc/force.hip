@@ -13,7 +13,7 @@
 namespace csph
 {
 
-
+// hsqinv, pres and auterm are the mixed form's (nullptr in FP64, which forms them where it needs them).
 __global__ __launch_bounds__(256) void forcePrepKernel(const double* __restrict__ h, const double* __restrict__ gradh,
                                                        const double* __restrict__ pro2, double* __restrict__ hsqinv,
                                                        double* __restrict__ hinv, double* __restrict__ rhoh,
@@ -28,8 +28,11 @@ __global__ __launch_bounds__(256) void forcePrepKernel(const double* __restrict_
     const double hi = h[i];
     if (!(hi > 0.0))
     {
-        hsqinv[i] = 0.0; hinv[i] = 0.0; rhoh[i] = 0.0; rho1[i] = 0.0; grkfac[i] = 0.0;
-        pres[i] = 0.0; auterm[i] = 0.0; divfac[i] = 0.0;
+        hinv[i] = 0.0; rhoh[i] = 0.0; rho1[i] = 0.0; grkfac[i] = 0.0; divfac[i] = 0.0;
+        if (hsqinv)
+        {
+            hsqinv[i] = 0.0; pres[i] = 0.0; auterm[i] = 0.0;
+        }
         return;
     }
     const double hs = 1.0 / (hi * hi), h4 = hs * hs, hfoh = hfact / hi;
@@ -37,14 +40,17 @@ __global__ __launch_bounds__(256) void forcePrepKernel(const double* __restrict_
     const double dhdrho = -hi / (3.0 * rho);
     const double omega = 1.0 - dhdrho * gradh[i];
     const double oinv = (omega > 0.0) ? (1 / omega) : 1.0;
-    hsqinv[i] = hs;
     hinv[i]   = 1.0 / hi;
     rhoh[i]   = rho;
     rho1[i]   = 1.0 / rho;
     grkfac[i] = h4 * kCnormk * oinv;
-    pres[i]   = pro2[i] * rho * rho;
-    auterm[i] = 0.5 * pmass * (1.0 / rho) * alphau;
     divfac[i] = kCnormk * oinv * h4 / rho;
+    if (hsqinv)
+    {
+        hsqinv[i] = hs;
+        pres[i]   = pro2[i] * rho * rho;
+        auterm[i] = 0.5 * pmass * (1.0 / rho) * alphau;
+    }
 }
 
 // A double of lane p as a scalar (p wave-uniform).  With every lane active: a register that was spilled

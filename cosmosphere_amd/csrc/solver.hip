@@ -428,9 +428,11 @@ ForceTimings computeForces(State& s, double pmass, double beta, double alphau, b
             std::fprintf(stderr, "WARNING! buildForceJLeafList: jlist_trunc=%d stack_drops=%d\n", hovf[0], hovf[1]);
     }
     e1.rec(st);
-    launchForcePrep(s.h.as<double>(), s.gradh.as<double>(), s.pro2.as<double>(), s.hsqinv.as<double>(),
+    const bool mixed = s.precision == kMixed;
+    launchForcePrep(s.h.as<double>(), s.gradh.as<double>(), s.pro2.as<double>(), mixed ? s.hsqinv.as<double>() : nullptr,
                     s.hinv.as<double>(), s.rhoh.as<double>(), s.rho1.as<double>(), s.grkfac.as<double>(),
-                    s.pres.as<double>(), s.auterm.as<double>(), s.divfac.as<double>(), n, pmass, alphau, s.hfact, st);
+                    mixed ? s.pres.as<double>() : nullptr, mixed ? s.auterm.as<double>() : nullptr,
+                    s.divfac.as<double>(), n, pmass, alphau, s.hfact, st);
     e2.rec(st);
     unsigned long long* ctr = zeroCounters(s);
     ForceArgs a{};
@@ -460,7 +462,6 @@ ForceTimings computeForces(State& s, double pmass, double beta, double alphau, b
     a.lbox = s.leafBox.as<double>(); a.lboxN = s.leafCap;
     a.sx = s.nodeSx.as<double>(); a.sy = s.nodeSy.as<double>(); a.sz = s.nodeSz.as<double>();
     a.hmaxLeaf = s.hmaxLeaf.as<double>();
-    const bool mixed = s.precision == kMixed;
     if (mixed)
     {
         a.f32Stride = (size_t)n + 1;
