@@ -218,10 +218,10 @@ def fp64_closure_reference(lib, c):
     return lib.array("h"), lib.array("rho")
 
 
-def build_oracle(c):
+def build_oracle(c, bucket=64):
     """The FP64 oracle's tree of the workload (keys, sort, leaf tree), timed."""
     from oracle import oracle as O
-    o = O.Oracle(quintic=c["quintic"])
+    o = O.Oracle(quintic=c["quintic"], bucket=bucket)
     o.set_particles(c["x"], c["y"], c["z"], c["h"])
     t = time.perf_counter()
     o.build()
@@ -274,28 +274,18 @@ def cpu_baseline(c, o, t_tree, gpu_h_fp64, gpu_h_mixed, seconds):
     return base, err
 
 
-def parity_full(lib, c, o, sample):
-    """Full-size parity against the FP64 oracle (the GPU's plain FP64 path, the oracle's tree):
-    keys, order, leaf tree and layout bit for bit; the all-leaf gather lists at the GPU's
-    converged h (one FP64 solve with the gradient sweep over gather lists, grad_sym_lists=0)
-    bit for bit; h and
-    rho of the sampled leaves' particles (the cpu_baseline sample), with the particles whose
-    Newton iteration stopped one step apart counted separately (|dh/h| above 1e-12: summation
-    order alone moves h by rounding, about 1e-15; a |dh/h| < tolh decision that rounding tipped
-    moves it by one Newton step, and rho, taken at the h before the last update, further: |drho/rho|
-    above 1e-10 marks such a particle too)."""
-    t0 = time.perf_counter()
-    lib.set_option("precision", 0)
-    lib.set_option("closure", -1)
+def parity_tree(lib, c, o, bucket):
+    """Keys, order, leaf tree and layout of an FP64 solve with the given leaf bucket, and the all-leaf
+    gather lists at its converged h, against the oracle's tree of that bucket, bit for bit."""
+    sym, was = lib.stat("grad_sym_lists"), lib.stat("bucket")
     lib.restore_inputs()
-    sym, bucket = lib.stat("grad_sym_lists"), lib.stat("bucket")
     lib.set_option("grad_sym_lists", 0)
-    lib.set_option("bucket", 64)   # the oracle's tree (the timed solves may be tuned to another)
+    lib.set_option("bucket", bucket)
     try:
         lib.solve_dens_h(c["n"], c["pmass"], 0, True, None, 1e-4, c["hfact"])
     finally:
         lib.set_option("grad_sym_lists", sym)
-        lib.set_option("bucket", int(bucket))
+        lib.set_option("bucket", int(was))
     out = {}
     cmp = {"keys": "keys", "order": "order", "leafLevel": "leafLevel", "layout": "layout"}
     for g, r in cmp.items():
@@ -311,8 +301,29 @@ def parity_full(lib, c, o, sample):
     ro, rl = o.get("jOffset"), o.get("jList")
     out["gather_lists"] = bool(jo.size == ro.size and np.array_equal(jo.astype(np.int64), ro.astype(np.int64))
                                and np.array_equal(jl, rl))
+    out["bit_exact"] = all(out.values())
     out["list_entries"] = int(rl.size)
     out["leaves"] = int(o.geti("nLeaves"))
+    return out
+
+
+def parity_full(lib, c, o, sample):
+    """Full-size parity against the FP64 oracle (the GPU's plain FP64 path): parity_tree on the
+    oracle's bucket of 64 and, where the timed solves are tuned to another, on theirs; h and
+    rho of the sampled leaves' particles (the cpu_baseline sample), with the particles whose
+    Newton iteration stopped one step apart counted separately (|dh/h| above 1e-12: summation
+    order alone moves h by rounding, about 1e-15; a |dh/h| < tolh decision that rounding tipped
+    moves it by one Newton step, and rho, taken at the h before the last update, further: |drho/rho|
+    above 1e-10 marks such a particle too)."""
+    t0 = time.perf_counter()
+    lib.set_option("precision", 0)
+    lib.set_option("closure", -1)
+    bucket = int(lib.stat("bucket"))
+    out = parity_tree(lib, c, o, 64)
+    exact = out.pop("bit_exact")
+    if bucket != 64:
+        out["timed_tree"] = dict(parity_tree(lib, c, build_oracle(c, bucket)[0], bucket), bucket=bucket)
+        exact = exact and out["timed_tree"]["bit_exact"]
     idx, h_ref, rho_ref = sample["sample_idx"], sample["sample_h"], sample["sample_rho"]
     h_fp64, rho_fp64 = sample["gpu_h_fp64_sorted"], sample["gpu_rho_fp64_sorted"]
     eh = np.abs(h_fp64[idx] - h_ref) / h_ref
@@ -327,7 +338,7 @@ def parity_full(lib, c, o, sample):
     out["sample_max_rel_err_rho_unflipped"] = float(er[~flip].max()) if (~flip).any() else 0.0
     out["sample_max_rel_err_h"] = float(eh.max())
     out["seconds"] = time.perf_counter() - t0
-    out["bit_exact"] = all(out[k] for k in ("keys", "order", "leafLevel", "layout", "leafStart", "gather_lists"))
+    out["bit_exact"] = exact
     return out
 
 
