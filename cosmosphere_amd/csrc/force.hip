@@ -85,7 +85,7 @@ __device__ inline double pressureOf(double pro2, double rho)
 // times those of a sum for each side.  The tile
 // holds what the pair needs of j; the pressure and the conductivity factor are taken from rho,
 // 1/rho and p/rho^2 rather than gathered (15 fields instead of 18).  The open instances fit four
-// wavefronts per SIMD (128 VGPRs, 9 KB of LDS each): the chunk's positions are read from their
+// wavefronts per SIMD (128 VGPRs, 9.5 KB of LDS each): the chunk's positions are read from their
 // owner lanes, its box sits in scalars.  The periodic ones, whose box fills
 // the scalars, keep positions in LDS and run three (0.61 ms; 0.66-0.70 by any of the other ways).
 // 1M-particle mixture, 1.31e8 pairs: 6.5 -> 4.9 ms (five sixths of it the pair terms); periodic box of
@@ -100,7 +100,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(PER ? 1 :
     // (a j is accepted by several particles of the chunk: reading its fields per pair would
     // be one scattered load per field per pair)
     // R2: the square of j's reach (R h)^2 (1 + 1e-10), or with DISC its h
-    enum { X, Y, Z, R2, VX, VY, VZ, HI, GK, RH, R1, P2, CS, AL, U, NF };
+    enum { X, Y, Z, R2, VX, VY, VZ, HS, HI, GK, RH, R1, P2, CS, AL, U, NF };
     __shared__ double tf[NF][kWave];
     __shared__ int    jq[2 * kWave];  // candidates that passed the particle test
     __shared__ double cp[4][PER ? kWave : 1];   // periodic: the chunk's particles: x, y, z, R h
@@ -126,7 +126,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(PER ? 1 :
             const double rhoi = A.rhoh[i], gki = A.grkfac[i], hinvi = A.hinv[i];
             const double pro2i = A.pro2[i], vwi = A.cs[i], ali = A.alpha[i], eni = A.u[i];
             const double rho1i = A.rho1[i], pri = pressureOf(pro2i, rhoi);
-            const double reach2 = kRad2 * (hi_ * hi_) * (1.0 + 1e-10);
+            const double reach2 = kRad2 * (hi_ * hi_) * (1.0 + 1e-10), hsi = 1.0 / (hi_ * hi_);
             double cbc[3], cbs[3], rChunk;   // the chunk's bounding box and largest reach R h
             const uint32_t ic = q0 + (uint32_t)(lane < c ? lane : 0);
             const double xc = A.x[ic], yc = A.y[ic], zc = A.z[ic], rc = kRad * A.h[ic];   // particle `lane` of the chunk
@@ -187,6 +187,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(PER ? 1 :
                 const double hj = A.h[j];
                 tf[X][l] = A.x[j]; tf[Y][l] = A.y[j]; tf[Z][l] = A.z[j];
                 tf[R2][l] = DISC ? hj : reachOf(hj);
+                tf[HS][l] = 1.0 / (hj * hj);   // (a division for a slot costs less than one more gather)
                 tf[VX][l] = A.vx[j]; tf[VY][l] = A.vy[j]; tf[VZ][l] = A.vz[j];
                 tf[HI][l] = A.hinv[j]; tf[GK][l] = A.grkfac[j];
                 tf[RH][l] = A.rhoh[j]; tf[R1][l] = A.rho1[j]; tf[P2][l] = A.pro2[j];
@@ -221,7 +222,9 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(PER ? 1 :
                 double dr, rij1;
                 sqrtAndInverse(dr2, dr, rij1);
                 const double qi = dr * hinvi, qj = dr * tf[HI][k];
-                const bool inI = qi < kRad, inJ = qj < kRad;
+                // in a support: rounded as the reference's r^2 / h^2 < R^2 (pairs at its edge count for the
+                // signal speed or do not)
+                const bool inI = dr2 * hsi < kRad2, inJ = dr2 * tf[HS][k] < kRad2;
                 rx = dx * rij1; ry = dy * rij1; rz = dz * rij1;
                 const double dvx = vxi - tf[VX][k], dvy = vyi - tf[VY][k], dvz = vzi - tf[VZ][k];
                 const double projv = dvx * rx + dvy * ry + dvz * rz;
