@@ -143,7 +143,8 @@ __device__ inline bool nearEps(double r)
 // The sweep waits on its gathers more than on arithmetic: the open-box mixed instance runs five
 // wavefronts per SIMD (96 VGPRs, 6 spilled); the others keep four.  FP64: pair terms by kernED and
 // one root for r and 1/r, 3.23 -> 2.78 ms on a carried step of the 1M-particle mixture, 0.61 -> 0.54
-// on a periodic box of 369k (then 2.31 and 0.43 with a wavefront to a block, sweepItem).
+// on a periodic box of 369k (then 2.31 and 0.43 with a wavefront to a block, sweepItem; 2.65 and 0.46 since
+// dW/dq is exact to the smallest q and near pairs have their reciprocal, 0.15 ms of it the branch for them).
 template<bool PER, bool MIXED>
 __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(MIXED && !PER ? 5 : 4))) void gradientKernel(GradArgs A)
 {

@@ -89,7 +89,9 @@ __device__ inline double pressureOf(double pro2, double rho)
 // owner lanes, its box sits in scalars.  The periodic ones, whose box fills
 // the scalars, keep positions in LDS and run three (0.61 ms; 0.66-0.70 by any of the other ways).
 // 1M-particle mixture, 1.31e8 pairs: 6.5 -> 4.9 ms (five sixths of it the pair terms); periodic box of
-// 369k: 0.87 -> 0.61 ms (then 3.85 and 0.55 with a wavefront to a block, sweepItem).
+// 369k: 0.87 -> 0.61 ms (then 3.85 and 0.55 with a wavefront to a block, sweepItem; 4.3 and 0.58 since dW/dq is
+// exact to the smallest q, sums are kept per tile and terms that are not finite are taken by sides;
+// 8 to 23 VGPRs spilled in the open instances).
 template<bool PER, bool DISC, bool FULL>
 __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(PER ? 1 : 4))) void forceKernel(ForceArgs A)
 {

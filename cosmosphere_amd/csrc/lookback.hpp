@@ -1,5 +1,6 @@
 /*
- * lookback.hpp -- the pieces of single-launch scans (decoupled look-back), shared by the scan
+ * lookback.hpp -- the pieces of single-launch scans (decoupled look-back: Merrill and Garland,
+ * "Single-pass Parallel Prefix Scan with Decoupled Look-back", 2016), shared by the scan
  * (prims.hip) and the compaction of the device-driven loop (loop.hip).
  *
  * A block's tile is taken from a counter, in the order the blocks start.  It publishes its tile's

@@ -10,7 +10,9 @@
  * 64 coalesced loads.  Wave-level multisplit: 8 ballots give each lane the mask of lanes with
  * its digit, the rank is the popcount below it, and a per-wave LDS counter carries ranks across
  * rounds -- so the order within a digit is the input order, which is what makes the sort stable.
- * The base of (digit, tile) comes from looking back over the earlier tiles' published counts.
+ * The base of (digit, tile) comes from looking back over the earlier tiles' published counts
+ * (the scheme of Adinets and Merrill, "Onesweep: A Faster Least Significant Digit Radix Sort for
+ * GPUs", 2022).
  */
 #include "density.hpp"
 #include "lookback.hpp"
