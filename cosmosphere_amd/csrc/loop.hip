@@ -98,7 +98,7 @@ struct QueueRule
 // kMaxSub: list ranges of one particle's items and of FP64 whole leaves, every n-th tile of mixed whole
 // leaves (each sub-item stages all of them, so n is bounded by the particles that the staging serves).
 // Density kernels of a solve without and with it: that disc (mixed) 13.3 and 8.4 ms, 12 sets of
-// 10k-60k particles 4.1 and 3.3 ms, a 2M-particle mixture 169 and 161 ms, a step of 1M 3.7 and 2.4 ms;
+// 10k-53k particles 4.1 and 3.3 ms, a 2M-particle mixture 169 and 161 ms, a step of 1M 3.7 and 2.4 ms;
 // items all alike (lattices) are not touched.
 //
 // Called by whole wavefronts (`is`: the lane has an item): one atomic per wavefront and counter.

@@ -21,7 +21,7 @@ constexpr size_t kListSlotWords = size_t(1) << 30;   // ... of all lists togethe
 // copying its tokens, so a slot is as long as the leaves' number allows (the first passes of a solve
 // have the longest lists: 1,900 entries on the 8M-particle mixture).  Lists of a solve with slots of
 // 256, 512, 1024, 2048 tokens: 250k-particle disc 5.2, 4.1, 3.7, 3.7 ms; 2M-particle mixture 19.1,
-// 18.4, 15.9, 14.5; 8M 75, 75, 73, 45; 12 sets of 10k-60k 2.7, 2.3, 2.3, 2.3.
+// 18.4, 15.9, 14.5; 8M 75, 75, 73, 45; 12 sets of 10k-53k 2.7, 2.3, 2.3, 2.3.
 inline int listSlotTokens(int leafCap)
 {
     int n = kListSlotMax;
